@@ -541,6 +541,179 @@ SZP_HD int parse_true_walk(const uint8_t *tb, const uint32_t *spec, uint32_t *pr
     return 0;
 }
 
+// ---- synchronised boundaries of the fused parse and decode ----
+//
+// The fused kernel cuts a chunk's block area (blocks in mode 1, units in mode
+// 2) into byte tiles of S bytes and each tile into sections.  For a section
+// starting at byte u, every chain that could be the true one starts in
+// [u, u + W) (W = longest step).  Chains that meet a width byte > 32 end; at a
+// horizon X the others have each a first position at or past X, and when they
+// agree on it, it lies on the true chain whatever precedes it: the section's
+// boundary, which the section that ends there and the one that starts there
+// find alone, from the same bytes.  The first horizon is u + 2 W, the last
+// u + V.  A section whose chains are still apart at u + V, or meet the first
+// horizon at more positions than it has lanes, has no boundary, and its
+// predecessor walks through it.  A boundary lies in [u + 2 W, u + V + W), and sections are at
+// least V bytes, so boundaries are in order.
+struct FusedShape {
+    uint32_t S;     // bytes of a tile
+    uint32_t W;     // longest step
+    uint32_t V;     // last horizon of a boundary
+    uint32_t nsec;  // sections of a tile
+    uint32_t sec;   // bytes of a section (the last one takes the remainder)
+    uint32_t ll;    // log2 of the lanes that look for one boundary
+    uint32_t per;   // candidates of a lane
+    uint32_t L;     // values of a full block (mode 2: of a full unit's block)
+    uint32_t c0;    // step of a block of width b > 0: c0 + ceil(b L / 8)
+};
+constexpr uint32_t kFusedMaxTile = 14336;
+constexpr uint32_t kFusedMinB = 8, kFusedMaxB = 256;
+constexpr uint32_t kFusedMaxSec = 15;
+constexpr uint32_t kFusedNone = 0xFFFFFFFFu;
+
+// The shape for streams of at most len bytes; false when the fused kernel
+// does not serve the geometry.  B from 8 to 256: longer blocks leave too few
+// of them in a tile for chains to meet, shorter ones make the walks long.
+// V = 6 W: a chain started off a block start survives a step with probability
+// about 1/3 on simulation data (many plane bytes are small) and its steps are
+// W / 2 on average, so ~11 steps leave less than one such chain among W
+// candidates in 100 sections (measured on a k^-3 field at REL 1e-4: without a
+// boundary are 91 % of sections at 3 W, 13 % at 4 W, 0.4 % at 6 W).  A
+// tile's bytes: 14 KiB (seven workgroups' LDS per CU at B = 128), halved while
+// the stream has fewer than 2048 tiles (small streams: all CUs work, and the
+// serial walks are short) or while a tile would hold more than 64 Ki values
+// (sparse streams: one workgroup writes a tile's values), but at least V.
+inline bool fused_shape(const Geom &g, uint64_t len, FusedShape *f)
+{
+    if (g.B < kFusedMinB || g.B > kFusedMaxB || g.n == 0) return false;
+    if (g.nb0 >= (1ull << 30) || g.nblast >= (1ull << 30)) return false;
+    f->L = g.mode == 2 ? g.B - 1 : g.B;
+    f->c0 = (g.mode == 2 ? 5 : 1) + (f->L + 7) / 8;
+    f->W = f->c0 + 4 * f->L;
+    f->V = 6 * f->W;
+    uint64_t S = kFusedMaxTile;
+    while (S / 2 >= f->V && S > 1792 && (len < S * 2048 || (g.n / 65536) * S > len)) S /= 2;
+    f->S = (uint32_t)S;
+    const uint32_t want = g.B >= 128 ? 3u : g.B >= 64 ? 7u : kFusedMaxSec;
+    const uint32_t most = f->S / f->V;
+    f->nsec = want < most ? want : most;
+    if (f->nsec == 0) return false;
+    f->sec = f->S / f->nsec;
+    f->ll = f->nsec < 4 ? 6u : f->nsec < 8 ? 5u : 4u;  // all boundaries at once
+    f->per = (f->W + (1u << f->ll) - 1) >> f->ll;
+    return true;
+}
+
+// LDS of a fused tile: the bytes staged (S + V + W + 16, up to 15 before them
+// and 16 of the last vector, and the 32 bytes the decode may read past a
+// block), and the bitmap's words.
+SZP_HD uint32_t fused_buf_bytes(const FusedShape &f) { return (f.S + f.V + f.W + 128) & ~15u; }
+SZP_HD uint32_t fused_bitmap_words(const FusedShape &f) { return (f.S + f.V + f.W) / 32 + 2; }
+
+SZP_HD uint32_t load_u32(const uint8_t *p)
+{
+    uint32_t w;
+    __builtin_memcpy(&w, p, 4);
+    return w;
+}
+
+// One step of a chain from p (p < end): a block or unit, or in mode 1 a run of
+// up to 3 zero blocks (single zero bytes), k of them, ending at `end` at most.
+// Returns the step's bytes; b > 32: no step starts here.  Reads 4 bytes at the
+// width byte.
+template <int MODE>
+SZP_HD uint32_t fused_step(const uint8_t *tb, uint32_t p, uint32_t end, const FusedShape &f,
+                           uint32_t &b, uint32_t &k)
+{
+    const uint32_t w = load_u32(tb + p + (MODE == 2 ? 4 : 0));
+    b = w & 255u;
+    uint32_t z = 1;
+    if (MODE == 1) {
+        const uint32_t run = (uint32_t)__builtin_ctz(w | 0x80000000u) >> 3;  // zero bytes, b = 0: 1 .. 3
+        z = run < end - p ? run : end - p;
+    }
+    k = b ? 1u : z;
+    return b ? f.c0 + ((b * f.L + 7) >> 3) : (MODE == 2 ? 5u : z);
+}
+
+// Which of the four bytes of w are at most 32 -- and not zero, with
+// NONZERO -- as bits 0-3.
+template <bool NONZERO>
+SZP_HD uint32_t bytes_le32(uint32_t w)
+{
+    // Bit 7 of a byte of t is set when the byte is over 32, of z when it is not 0.
+    const uint32_t lo = w & 0x7F7F7F7Fu;
+    const uint32_t t = (lo + 0x5F5F5F5Fu) | w, z = (lo + 0x7F7F7F7Fu) | w;
+    const uint32_t v = ((NONZERO ? ~t & z : ~t) >> 7) & 0x01010101u;
+#ifdef __HIP_DEVICE_COMPILE__
+    return __builtin_amdgcn_udot4(v, 0x08040201u, 0u, false);
+#else
+    return (v & 1) | ((v >> 7) & 2) | ((v >> 14) & 4) | ((v >> 21) & 8);
+#endif
+}
+
+// Candidates [c, cend), at most f.per of them: walks the chain of each to X
+// and hands its first position at or past X to `keep` when it gets there.  The
+// first width bytes are tested four at a time; most candidates end there.  A
+// zero block (mode 1) is one byte long, so its chain is the next candidate's:
+// of those only the last candidate of all (lastc) is walked.
+template <int MODE, typename KEEP>
+SZP_HD void sync_walk(const uint8_t *tb, uint32_t c, uint32_t cend, uint32_t lastc, uint32_t X,
+                      const FusedShape &f, KEEP keep)
+{
+    for (uint32_t k0 = 0; k0 < f.per; k0 += 32) {
+        uint32_t m = 0;
+        for (uint32_t k = 0; k < 32 && k0 + k < f.per; k += 4)
+            m |= bytes_le32<MODE == 1>(load_u32(tb + c + k0 + k + (MODE == 2 ? 4 : 0))) << k;
+        const uint32_t left = c + k0 < cend ? cend - (c + k0) : 0u;
+        if (left < 32) m &= (1u << left) - 1u;
+        if (MODE == 1 && lastc - (c + k0) < (left < 32 ? left : 32u) && tb[lastc] == 0)
+            m |= 1u << (lastc - (c + k0));
+        uint32_t p = X;
+        while (true) {
+            if (p >= X) {
+                if (!m) break;
+                p = c + k0 + (uint32_t)__builtin_ctz(m);
+                m &= m - 1;
+            }
+            uint32_t b, k;
+            const uint32_t len = fused_step<MODE>(tb, p, X, f, b, k);
+            p = b > 32 ? X : p + len;
+            if (b <= 32 && p >= X) keep(p);
+        }
+    }
+}
+
+// One chain that is left, from p to X (kFusedNone when it ends before).
+template <int MODE>
+SZP_HD uint32_t sync_more(const uint8_t *tb, uint32_t p, uint32_t X, const FusedShape &f)
+{
+    while (p < X) {
+        uint32_t b, k;
+        const uint32_t len = fused_step<MODE>(tb, p, X, f, b, k);
+        p = b > 32 ? kFusedNone : p + len;
+    }
+    return p;
+}
+
+// The true chain of a section from p up to `end`: marks its starts in bm.
+// Returns false when it meets a width byte > 32 (p stays there).
+template <int MODE, typename OR = BmOr>
+SZP_HD bool fused_walk(const uint8_t *tb, uint32_t *bm, uint32_t &p, uint32_t end,
+                       const FusedShape &f, OR op = OR())
+{
+    while (p < end) {
+        uint32_t b, k;
+        const uint32_t len = fused_step<MODE>(tb, p, end, f, b, k);
+        if (b > 32) return false;
+        const uint32_t bits = (1u << k) - 1u, sh = p & 31;
+        op(&bm[p >> 5], bits << sh);
+        if (sh + k > 32) op(&bm[(p >> 5) + 1], bits >> (32 - sh));
+        p += len;
+    }
+    return true;
+}
+
 // Rank of p among the set bits of bm within its sub-tile (rk holds, per word,
 // the set bits of the sub-tile's earlier words).
 SZP_HD uint32_t parse_rank(const uint32_t *bm, const uint16_t *rk, uint32_t p)

@@ -729,6 +729,9 @@ __global__ void k_empty_stream(uint8_t *out, const V *d_eb, V eb_host, uint32_t 
     }
 }
 
+// A value that is the same in every lane, as a scalar register.
+__device__ __forceinline__ uint32_t uniform(uint32_t v) { return __builtin_amdgcn_readfirstlane(v); }
+
 // Unaligned LDS accesses (gfx950 runs with unaligned LDS access enabled; the
 // compiler emits ds_read/ds_write_b32/b64/b128 for these copies).
 __device__ __forceinline__ void lds_st32(uint8_t *p, uint32_t v) { __builtin_memcpy(p, &v, 4); }
@@ -2234,6 +2237,92 @@ __device__ __forceinline__ uint32_t decode_slot(uint32_t L, bool head, uint32_t 
     return m;
 }
 
+// Residuals and signs of a full octet of plane values v (mag >> r): res holds
+// the 8 r-bit residuals MSB-first, sg the signs MSB-first.  SUM: returns the
+// sum of the deltas (dl is not written); otherwise dl[i] is their inclusive
+// prefix.  A residual is one bit-field extract of a 32-bit half (the halves
+// hold four each, 4r <= 28 bits), a magnitude one shift-or, a signed one
+// (mag ^ s) - s with s = 0 or -1; no 64-bit shifts, no multiplies.
+template <bool SUM>
+__device__ __forceinline__ uint32_t octet_signed(const uint32_t v[8], uint32_t r, uint2 res,
+                                                 uint32_t sg, uint32_t dl[8])
+{
+    const uint32_t h = __builtin_bswap32(res.x);
+    // The next four values, from the top bit (r = 0: any, no bits are taken).
+    const uint32_t l = __builtin_amdgcn_alignbit(h, __builtin_bswap32(res.y), 32u - 4u * r);
+    uint32_t run = 0;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+        const uint32_t low = __builtin_amdgcn_ubfe(i < 4 ? h : l, 32u - r * (uint32_t)(i % 4 + 1), r);
+        const uint32_t mag = (v[i] << r) | low;
+        const uint32_t s = (uint32_t)__builtin_amdgcn_sbfe((int)sg, 7 - i, 1);
+        run = (mag ^ s) + run;
+        if (!SUM) {
+            run -= s;
+            dl[i] = run;
+        }
+    }
+    return SUM ? run + (uint32_t)__builtin_popcount(sg) : run;
+}
+
+// Unpacks octet o of a block at buf[lp] of L = 8 * spb values (a unit's block:
+// L = 8 * spb - 1, where the last octet's eighth delta is not one and dl[7]
+// is not used), of width b <= 32 and with all its bytes present: the deltas'
+// inclusive prefix in dl, or with SUM only their sum; returns the sum.  When no lane of the wave has
+// a width over 15 (at most one plane byte) it takes a path without branches.
+// (A b = 0 block's "sign byte" belongs to what follows it, which is harmless:
+// its magnitudes are zero.)
+template <bool SUM>
+__device__ __forceinline__ uint32_t decode_octet8(const uint8_t *buf, uint32_t lp, uint32_t b,
+                                                  uint32_t spb, uint32_t L, uint32_t o,
+                                                  uint32_t dl[8])
+{
+    const uint32_t sg = buf[lp + 1 + o];
+    const uint32_t nb = b >> 3, r = b & 7;
+    const uint8_t *pb = buf + lp + 1 + spb;
+    const uint8_t *p1 = pb + __umul24(8 * o, nb);
+    const uint2 res = lds_ld64(pb + __umul24(L, nb) + __umul24(o, r));
+    uint32_t v[8];
+    if (__ballot(nb > 1) == 0) {
+        uint2 w = lds_ld64(p1);
+        w.x = nb ? w.x : 0u;
+        w.y = nb ? w.y : 0u;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            v[i] = __builtin_amdgcn_ubfe(w.x, 8 * i, 8);
+            v[i + 4] = __builtin_amdgcn_ubfe(w.y, 8 * i, 8);
+        }
+        return octet_signed<SUM>(v, r, res, sg, dl);
+    }
+    const uint4 a = lds_ld128(p1), c = lds_ld128(p1 + 16);
+    // Byte offsets nb * i of the octet's 8 nb plane bytes, as shifts of pairs
+    // of their words.
+    const uint32_t m = nb == 4 ? ~0u : (1u << (8 * nb)) - 1u;
+    if (nb < 2) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            v[i] = (a.x >> (8 * i)) & m & 0xFFu;
+            v[i + 4] = (a.y >> (8 * i)) & m & 0xFFu;
+        }
+    } else if (nb == 2) {
+        v[0] = a.x & m; v[1] = a.x >> 16; v[2] = a.y & m; v[3] = a.y >> 16;
+        v[4] = a.z & m; v[5] = a.z >> 16; v[6] = a.w & m; v[7] = a.w >> 16;
+    } else if (nb == 3) {
+        v[0] = a.x & m;
+        v[1] = __builtin_amdgcn_alignbyte(a.y, a.x, 3) & m;
+        v[2] = __builtin_amdgcn_alignbyte(a.z, a.y, 2) & m;
+        v[3] = a.z >> 8;
+        v[4] = a.w & m;
+        v[5] = __builtin_amdgcn_alignbyte(c.x, a.w, 3) & m;
+        v[6] = __builtin_amdgcn_alignbyte(c.y, c.x, 2) & m;
+        v[7] = c.y >> 8;
+    } else {
+        v[0] = a.x; v[1] = a.y; v[2] = a.z; v[3] = a.w;
+        v[4] = c.x; v[5] = c.y; v[6] = c.z; v[7] = c.w;
+    }
+    return octet_signed<SUM>(v, r, res, sg, dl);
+}
+
 // Segmented scan of slot aggregates (h, v) in slot order: a head restarts
 // the running value.  Returns the slot's exclusive (eh, ev) and the round's
 // total (rh, rv).
@@ -2775,6 +2864,568 @@ __global__ __launch_bounds__(kWG) void k_decode(const uint8_t *__restrict__ st, 
         return;
     }
     decode_tile<V, INDEXED, SPB>(st, len, g, blkpos, idx_carry, out, status, ctl, tile, L);
+}
+
+// ---------------------------------------------------------------------------
+// Fused parse and decode of a foreign stream
+// ---------------------------------------------------------------------------
+//
+// One workgroup takes a byte tile of a chunk's block area (szp_geom.h,
+// FusedShape) from stream bytes to values:
+//  1. The tile's bytes, and what its last blocks need beyond it, go to LDS.
+//  2. The waves find the boundaries of the tile's sections and of the next
+//     tile (sync_walk): positions on the true chain that depend on nothing
+//     before them, so a tile waits for its predecessor's exit only when its
+//     own boundary is missing.
+//  3. One lane per section walks the true chain from its boundary to the next
+//     and marks the block starts in a bitmap; the bitmap's ranks give the
+//     tile's block count and the list of positions.
+//  4. The waves unpack the blocks for the sum of their deltas; the tile
+//     publishes (block count, delta sum) in one word, and one grouped look-back
+//     gives the number of its first block, hence its elements, and its carry.
+//  5. Every wave unpacks its share of the blocks again, scans the deltas
+//     within the wave and writes the values.
+// Fast mode 2 restarts the chain in every unit: no sum is taken.
+//
+// What bounds it: latency (a tile's phases follow one another: staging and
+// boundaries ~105, walk ~48, sums ~53, look-back ~50, writing ~80 us of the
+// 512^3 field at REL 1e-4, B = 128) at 28 waves per CU, and in the unpacking
+// VALU issue.  Against a parse kernel that writes every block's position,
+// followed by a decode kernel that reads the stream again and looks back for
+// its carry: 480 -> 335 us on that field, 312 -> 213 us on a 384^3 float64
+// field (REL 1e-2, B = 64), 183 -> 133 us in fastMode 2 (384^3), 89 -> 29 us on
+// 100 003 values (B = 32).  Tiles of 11 and 20 KiB: 386 and 348 us.  Values go
+// out non-temporal in float (345 -> 335 us; double 213 -> 507 us).
+
+constexpr uint32_t kFusedSeg = 512;  // blocks whose positions are listed at a time
+
+// Sum of v over the wave, in every lane (DPP scan, no LDS permutes).
+__device__ __forceinline__ uint32_t wave_total_u32(uint32_t v)
+{
+    return __builtin_amdgcn_readlane(wave_incl_scan_u32(v, 0), 63);
+}
+// Least v of the lane's group of `lanes` lanes (a power of two from 16 to 64):
+// row_ror 8, 4, 2, 1 within a DPP row, then across rows.  A group's lanes are
+// all active or none is.
+__device__ __forceinline__ uint32_t group_min_u32(uint32_t v, uint32_t lanes)
+{
+    v = min(v, (uint32_t)__builtin_amdgcn_update_dpp(-1, (int)v, 0x128, 0xF, 0xF, false));
+    v = min(v, (uint32_t)__builtin_amdgcn_update_dpp(-1, (int)v, 0x124, 0xF, 0xF, false));
+    v = min(v, (uint32_t)__builtin_amdgcn_update_dpp(-1, (int)v, 0x122, 0xF, 0xF, false));
+    v = min(v, (uint32_t)__builtin_amdgcn_update_dpp(-1, (int)v, 0x121, 0xF, 0xF, false));
+    for (uint32_t o = 16; o < lanes; o <<= 1) v = min(v, (uint32_t)__shfl_xor((int)v, (int)o));
+    return v;
+}
+
+// Look-back words of the fused kernel: [flag 2][blocks 30][delta sum 32], the
+// two parts summed apart.  A chunk's first tile is absolute (inclusive from
+// the start).  own: each tile's first word, never overwritten (a group's last
+// tile sums them); st: the tile's current word; gst: one word per group of
+// kLbGroup tiles, kGroupStride words apart, inclusive from the group's last
+// absolute tile on.
+struct FusedStatus {
+    uint64_t *own, *st, *gst;
+};
+__device__ __forceinline__ uint64_t fused_word(uint64_t flag, uint32_t cnt, uint32_t sum)
+{
+    return flag | ((uint64_t)(cnt & 0x3FFFFFFFu) << 32) | sum;
+}
+
+// Sums of a wave's words up to and including its nearest inclusive one
+// (lanes ordered nearest first).
+__device__ __forceinline__ void fused_part(uint64_t w, bool &found, uint32_t &cnt, uint32_t &sum)
+{
+    const uint64_t m = __ballot((w >> 62) == 2);
+    const int f = m ? __ffsll((long long)m) - 1 : 64;
+    found = m != 0;
+    const bool in = __lane_id() <= f;
+    cnt = wave_total_u32(in ? (uint32_t)(w >> 32) & 0x3FFFFFFFu : 0u);
+    sum = wave_total_u32(in ? (uint32_t)w : 0u);
+}
+
+// Publishes a tile's first word (wave 0, all lanes) and, for a group's last
+// tile, the group's.
+__device__ __forceinline__ void fused_publish(const FusedStatus &S, uint64_t tile, uint64_t word,
+                                              uint32_t *ctl)
+{
+    const int lane = __lane_id();
+    if (lane == 0) {
+        st_status(&S.own[tile], word);
+        st_status(&S.st[tile], word);
+    }
+    if (tile % kLbGroup != kLbGroup - 1) return;
+    const uint64_t w = lane == 0 ? word : wait_status(&S.own[tile - lane], ctl);
+    bool found;
+    uint32_t cnt, sum;
+    fused_part(w, found, cnt, sum);
+    if (lane == 0)
+        st_status(&S.gst[(tile / kLbGroup) * kGroupStride],
+                  fused_word(found ? kFlagIncl : kFlagAgg, cnt, sum));
+}
+
+// Look-back of a tile that is not absolute, after fused_publish (all threads
+// call it): the blocks and the carry before it, in every thread; publishes
+// its inclusive word.  The same steps as lookback_compress.
+__device__ __forceinline__ void fused_lookback(const FusedStatus &S, uint64_t tile, uint32_t cnt,
+                                               uint32_t sum, uint32_t *ctl, uint64_t *s_lb,
+                                               uint32_t &pcnt, uint32_t &psum)
+{
+    const int tid = threadIdx.x, wv = tid >> 6, lane = __lane_id();
+    const uint64_t gr = tile / kLbGroup;
+    const uint32_t j = (uint32_t)(tile % kLbGroup);
+    pcnt = 0;
+    psum = 0;
+    bool done = false;
+    // The first step: this group's and the previous group's tiles (waves 0-1)
+    // and 128 groups before them; further steps: kWG groups each.
+    int64_t hi = (int64_t)gr - kLbRawWaves + 64 * kLbRawWaves;
+    for (uint32_t step = 0; !done; ++step) {  // uniform: every thread combines the same slots
+        uint64_t w;
+        if (step == 0 && wv < kLbRawWaves) {
+            const uint32_t back = (uint32_t)min<uint64_t>(gr, kLbRawWaves - 1) * kLbGroup;
+            w = (uint32_t)tid < j + back ? wait_status(&S.st[tile - 1 - tid], ctl) : 0;
+        } else {
+            const int64_t gi = hi - tid;
+            w = gi >= 0 ? wait_status(&S.gst[(uint64_t)gi * kGroupStride], ctl) : kFlagIncl;
+        }
+        bool found;
+        uint32_t c, v;
+        fused_part(w, found, c, v);
+        uint64_t *slot = s_lb + (step & 1) * 4;
+        if (lane == 0) slot[wv] = fused_word(found ? kFlagIncl : 0, c, v);
+        __syncthreads();
+#pragma unroll
+        for (int k = 0; k < kWG / 64; ++k) {
+            const uint64_t e = slot[k];
+            if (!done) {
+                pcnt += (uint32_t)(e >> 32) & 0x3FFFFFFFu;
+                psum += (uint32_t)e;
+                done = (e >> 62) == 2;
+            }
+        }
+        hi -= kWG;
+    }
+    pcnt &= 0x3FFFFFFFu;
+    if (tid == 0) {
+        const uint64_t inc = fused_word(kFlagIncl, pcnt + cnt, psum + sum);
+        st_status(&S.st[tile], inc);
+        if (j + 1 == kLbGroup) st_status(&S.gst[gr * kGroupStride], inc);
+    }
+}
+
+// Chunk table of the fused kernel, as k_dsetup's (ctab = [cstart | aend |
+// ttab]), by one workgroup with a scan over the chunks; a chunk that holds
+// values has at least one tile.  All workgroups clear the look-back words.
+__global__ __launch_bounds__(kWG) void k_fused_setup(const uint8_t *__restrict__ st, uint64_t len,
+                                                     Geom g, uint32_t S, uint64_t *__restrict__ ctab,
+                                                     uint64_t *__restrict__ clr, uint64_t nclr,
+                                                     uint32_t *__restrict__ ctl)
+{
+    for (uint64_t k = (uint64_t)blockIdx.x * kWG + threadIdx.x; k < nclr;
+         k += (uint64_t)gridDim.x * kWG)
+        clr[k] = 0;
+    if (blockIdx.x != 0) return;
+    __shared__ uint64_t s_w[kWG / 64];
+    __shared__ int s_bad;
+    const int tid = threadIdx.x, lane = __lane_id(), wv = tid >> 6;
+    if (tid < 8) ctl[tid] = 0;
+    if (tid == 0) s_bad = len < g.body;
+    __syncthreads();
+    uint64_t *cstart = ctab, *aend = ctab + g.T, *ttab = ctab + 2 * g.T;
+    uint64_t run = 0;
+    if (!s_bad) {
+        for (uint32_t t0 = 0; t0 < g.T; t0 += kWG) {
+            const uint32_t t = t0 + tid;
+            uint64_t tiles = 0;
+            if (t < g.T) {
+                const uint64_t nt = chunk_len(g, t);
+                const uint64_t off = read_u64_le4(st + g.es + 8ull * t);
+                const uint64_t nxt = t + 1 < g.T ? read_u64_le4(st + g.es + 8ull * (t + 1)) : 0;
+                const uint64_t cs = g.body + off;
+                uint64_t ce = cs;
+                bool bad = false;
+                if (nt == 0) {
+                    bad = off != 0;
+                } else {
+                    ce = t + 1 < g.T ? g.body + nxt : len;
+                    const uint64_t a0 = g.mode == 2 ? cs : cs + 4;
+                    bad = off > len || nxt > len || a0 + (g.mode == 2 ? 5 : 0) > ce || a0 > ce || ce > len;
+                    const uint64_t nb = t == g.T - 1 ? g.nblast : g.nb0;
+                    const uint64_t alen = bad ? 0 : ce - a0;
+                    bad = bad || (nb && !alen);
+                    tiles = nb && alen ? (alen + S - 1) / S : 1;
+                }
+                cstart[t] = cs;
+                aend[t] = ce;
+                if (bad) s_bad = 1;
+            }
+            uint64_t incl = tiles;
+#pragma unroll
+            for (int o = 1; o < 64; o <<= 1) {
+                const uint64_t v = __shfl_up(incl, o);
+                if (lane >= o) incl += v;
+            }
+            if (lane == 63) s_w[wv] = incl;
+            __syncthreads();
+            uint64_t before = run;
+            for (int k = 0; k < kWG / 64; ++k) {
+                if (k < wv) before += s_w[k];
+                run += s_w[k];
+            }
+            if (t < g.T) ttab[t] = before + incl - tiles;
+            __syncthreads();
+        }
+    }
+    __syncthreads();
+    if (s_bad) {
+        if (tid == 0) raise_error(ctl, kErrStream);
+        for (uint32_t t = tid; t < g.T; t += kWG) ttab[t] = 0;
+        run = 0;
+    }
+    if (tid == 0) ttab[g.T] = run;
+}
+
+template <typename V, int MODE, bool FULL8>
+__global__ __launch_bounds__(kWG, sizeof(V) == 4 ? 7 : 5) void k_fused_decode(
+    const uint8_t *__restrict__ st, uint64_t len, Geom g, FusedShape f, uint32_t nbuf,
+    uint32_t nword, const uint64_t *__restrict__ ctab, uint64_t *__restrict__ exit_st,
+    FusedStatus S, V *__restrict__ out, uint32_t *__restrict__ ctl)
+{
+    // LDS: the tile's bytes, the bitmap (nword words), the position list.
+    extern __shared__ __align__(16) uint8_t dyn[];
+    uint8_t *buf = dyn;
+    uint32_t *bm = reinterpret_cast<uint32_t *>(dyn + nbuf);
+    uint32_t *list = bm + nword;  // [no block 1][width 15][position 16]
+    __shared__ uint32_t s_bnd[kFusedMaxSec + 1], s_cnt[4], s_sum[4], s_brk;
+    __shared__ uint64_t s_lb[8];
+
+    const int tid = threadIdx.x, lane = __lane_id();
+    const uint32_t wv = uniform((uint32_t)tid >> 6);
+    const uint64_t gt = blockIdx.x;
+    const uint64_t *cstart = ctab, *aend = ctab + g.T, *ttab = ctab + 2 * g.T;
+    if (gt >= ttab[g.T]) return;
+    __builtin_amdgcn_s_setprio(2);  // until the tile's word is published
+    uint32_t t = 0;
+    {
+        uint32_t hi = g.T - 1;
+        while (t < hi) {
+            const uint32_t mid = (t + hi + 1) >> 1;
+            if (ttab[mid] <= gt) t = mid; else hi = mid - 1;
+        }
+    }
+    const uint64_t i = gt - ttab[t];
+    const bool first = i == 0;
+    const uint64_t cs = cstart[t], ae = aend[t];
+    const uint64_t s = cs + (MODE == 2 ? 0 : 4) + i * f.S;
+    const uint32_t span = (uint32_t)(min<uint64_t>(s + f.S, ae) - s);
+    const uint64_t s0 = s & ~15ull;
+    const uint32_t sh = (uint32_t)(s - s0);
+    const uint64_t tl = min<uint64_t>(s + f.S + f.V + f.W + 16, len);  // end of the staged bytes
+    const uint32_t B = g.B;
+    const uint64_t nbt = t == g.T - 1 ? g.nblast : g.nb0;
+
+    stage_bytes(st, len, s0, tl, buf);
+    for (uint32_t k = tid; k < nword; k += kWG) bm[k] = 0;
+    if (tid == 0) s_brk = kFusedNone;
+    if (tid <= (int)kFusedMaxSec) s_bnd[tid] = 0;
+    // The chunk's head (mode 1): its first value, and the chunk's carry.
+    uint32_t head = 0;
+    if (MODE == 1 && first) {
+        uint32_t v;
+        __builtin_memcpy(&v, st + cs, 4);
+        head = uniform(v);
+    }
+    __syncthreads();
+    const uint8_t *tb = buf + sh;  // tile byte p is tb[p]
+    const uint32_t lend = (uint32_t)(tl - s);
+
+    // Boundaries of the sections and of the next tile, all at once, 2^f.ll
+    // lanes each.  The positions at which chains meet the first horizon are
+    // listed once each (the bitmap tells which are; its bits are taken back).
+    {
+        const uint32_t b = (uint32_t)tid >> f.ll, r = (uint32_t)tid & ((1u << f.ll) - 1u);
+        const uint32_t u = b == f.nsec ? f.S : b * f.sec;
+        uint16_t *left = reinterpret_cast<uint16_t *>(list) + (b << f.ll);
+        const bool look = b <= f.nsec && !(b == 0 && first) && s + u + f.V <= ae &&
+                          s + u + f.V + 8 <= len;
+        uint32_t X = u + 2 * f.W;
+        if (look) {
+            const uint32_t c = min(u + f.per * r, u + f.W);
+            sync_walk<MODE>(tb, c, min(c + f.per, u + f.W), u + f.W - 1, X, f, [&](uint32_t q) {
+                const uint32_t bit = 1u << (q & 31);
+                if (atomicOr(&bm[q >> 5], bit) & bit) return;
+                const uint32_t k = atomicAdd(&s_bnd[b], 1u);
+                if (!(k >> f.ll)) left[k] = (uint16_t)q;
+            });
+        }
+        __syncthreads();
+        const uint32_t n = look ? s_bnd[b] : 0u;
+        for (uint32_t k = (X >> 5) + r; n && k <= (X + f.W) >> 5; k += 1u << f.ll) bm[k] = 0;
+        uint32_t P = kFusedNone;
+        uint32_t p = r < n && n <= 1u << f.ll ? left[r] : kFusedNone;
+        // Uniform in the group; one whose chains agree, have all ended or are
+        // too many is done.
+        while (true) {
+            const uint32_t least = group_min_u32(p, 1u << f.ll);
+            if (least == kFusedNone) break;
+            if (group_min_u32(p == kFusedNone ? kFusedNone : ~p, 1u << f.ll) == ~least) {
+                P = least;
+                break;
+            }
+            if (X == u + f.V) break;
+            X = min(X + f.W, u + f.V);
+            if (p != kFusedNone) p = sync_more<MODE>(tb, p, X, f);
+        }
+        if (b == 0 && first) P = 0;
+        if (r == 0 && b <= f.nsec) s_bnd[b] = P;
+    }
+    __syncthreads();
+
+    // The true chain, one lane per section.
+    if ((uint32_t)tid < f.nsec) {
+        uint32_t p = s_bnd[tid];
+        bool act = p != kFusedNone, broken = false;
+        if (tid == 0 && !act) {
+            const uint64_t e = wait_status(&exit_st[gt - 1], ctl) & kValMask;
+            broken = e < s;  // an exit before this tile: corrupt stream
+            p = broken ? 0 : (uint32_t)min<uint64_t>(e - s, f.S + f.W);
+            act = true;
+        }
+        if (act) {
+            uint32_t end = kFusedNone;
+            for (uint32_t k = tid + 1; k <= f.nsec && end == kFusedNone; ++k) end = s_bnd[k];
+            const bool open = end == kFusedNone;  // the chunk's last tile, or the next has no boundary
+            if (open) end = span;
+            if (!broken) broken = !fused_walk<MODE>(tb, bm, p, end, f, BmAtomicOr());
+            if (!open && p > end) broken = true;  // past a boundary: corrupt stream
+            if (broken) atomicMin(&s_brk, min(p, end));
+            if (open) st_status(&exit_st[gt], kFlagIncl | (broken ? s + span : s + p));
+        }
+    }
+    __syncthreads();
+
+    // Ranks: each thread owns up to wpt consecutive words of the bitmap.
+    const uint32_t wpt = (nword + kWG - 1) / kWG;
+    const uint32_t w0 = min(wpt * (uint32_t)tid, nword), w1 = min(w0 + wpt, nword);
+    uint32_t own = 0;
+    for (uint32_t k = w0; k < w1; ++k) own += (uint32_t)__builtin_popcount(bm[k]);
+    const uint32_t oincl = wave_incl_scan_u32(own, lane);
+    if (lane == 63) s_cnt[wv] = oincl;
+    __syncthreads();
+    uint32_t rank0 = oincl - own, tcnt = 0;
+#pragma unroll
+    for (uint32_t w = 0; w < kWG / 64; ++w) {
+        const uint32_t c = uniform(s_cnt[w]);
+        rank0 += w < wv ? c : 0u;
+        tcnt += c;
+    }
+    // Lists the positions of blocks [base, base + kFusedSeg) of the tile.
+    auto fill_list = [&](uint32_t base) {
+        uint32_t r = rank0;
+        for (uint32_t k = w0; k < w1; ++k) {
+            uint32_t m = bm[k];
+            while (m) {
+                const uint32_t bit = (uint32_t)__builtin_ctz(m);
+                m &= m - 1;
+                const uint32_t q = k * 32 + bit;
+                if (r - base < kFusedSeg) {
+                    // A block that is no block, or runs past the bytes
+                    // present, is listed as width 0 with the top bit set.
+                    const uint32_t b = tb[q + (MODE == 2 ? 4 : 0)];
+                    const uint32_t n = b ? f.c0 + ((b * f.L + 7) >> 3) : 1u;
+                    const bool ok = b <= 32 && q + n <= lend;
+                    list[r - base] = q | (ok ? b << 16 : 1u << 31);
+                }
+                ++r;
+            }
+        }
+    };
+    fill_list(0);
+    __syncthreads();
+
+    // A wave's step is KS blocks, spb lanes each; a segment's steps are split
+    // evenly over the waves, in order.
+    const uint32_t spb = g.spb, KS = 64 / spb;
+    const uint32_t ld = ((uint32_t)lane * g.spb_magic) >> 16, lo_ = (uint32_t)lane - ld * spb;
+    auto wave_steps = [&](uint32_t nb, uint32_t &a, uint32_t &z) {
+        const uint32_t steps = (nb + KS - 1) / KS;
+        a = steps * wv / 4;
+        z = steps * (wv + 1) / 4;
+    };
+    // Sum of the deltas of this wave's steps of a segment of nb blocks.
+    auto seg_sum = [&](uint32_t nb) -> uint32_t {
+        uint32_t a, z, acc = 0;
+        wave_steps(nb, a, z);
+        bool bad = false;  // reported by the writing pass, for blocks of the chunk
+        uint32_t dl[8];
+        uint32_t e = list[min(a * KS + ld, nb - 1)];
+        for (uint32_t q = a; q < z; ++q) {
+            const uint32_t j = q * KS + ld, en = list[min(j + KS, nb - 1)];  // the next step's entry
+            const bool act = ld < KS && j < nb;
+            if (FULL8) {
+                const uint32_t d = decode_octet8<true>(tb, e & 0xFFFFu, (e >> 16) & 63u, spb, B, lo_, dl);
+                acc += act ? d : 0u;
+            } else if (act) {
+                uint32_t h;
+                decode_slot(B, false, lo_, tb, e & 0xFFFFu, lend, dl, h, bad);
+                acc += dl[7];
+            }
+            e = en;
+        }
+        return wave_total_u32(acc);
+    };
+    uint32_t tsum = 0;
+    if (MODE == 1) {
+        for (uint32_t base = 0; base < tcnt; base += kFusedSeg) {
+            if (base) {
+                __syncthreads();
+                fill_list(base);
+                __syncthreads();
+            }
+            const uint32_t ws = seg_sum(min(tcnt - base, kFusedSeg));
+            if (tcnt <= kFusedSeg) {
+                if (lane == 0) s_sum[wv] = ws;
+            } else {
+                tsum += ws;
+            }
+        }
+        if (tcnt > kFusedSeg && lane == 0) s_sum[wv] = tsum;
+        if (tcnt == 0 && lane == 0) s_sum[wv] = 0;
+        __syncthreads();
+        tsum = 0;
+#pragma unroll
+        for (uint32_t w = 0; w < kWG / 64; ++w) tsum += uniform(s_sum[w]);
+    }
+
+    // Block number and carry of the tile.
+    uint32_t pcnt = 0, carry = head;
+    if (wv == 0)
+        fused_publish(S, gt, fused_word(first ? kFlagIncl : kFlagAgg, tcnt, tsum + head), ctl);
+    __builtin_amdgcn_s_setprio(0);
+    if (!first) {
+        fused_lookback(S, gt, tcnt, tsum, ctl, s_lb, pcnt, carry);
+        pcnt = uniform(pcnt);
+        carry = uniform(carry);
+    }
+
+    // A chain that broke before the chunk's last block, or a chunk that ends
+    // short of it, is malformed.
+    bool bad = false;
+    const uint32_t brk = uniform(s_brk);
+    if (brk != kFusedNone) {
+        uint32_t c = 0;
+        for (uint32_t k = w0; k < w1; ++k)
+            if (k * 32 < brk) c += (uint32_t)__builtin_popcount(bm[k] & bm_mask(k, 0, brk));
+        if (lane == 0) s_cnt[wv] = 0;
+        __syncthreads();
+        c = wave_total_u32(c);
+        if (lane == 0) s_cnt[wv] = c;
+        __syncthreads();
+        bad = (uint64_t)pcnt + s_cnt[0] + s_cnt[1] + s_cnt[2] + s_cnt[3] < nbt;
+    }
+    if (gt + 1 == ttab[t + 1] && (uint64_t)pcnt + tcnt < nbt) bad = true;
+    const uint32_t nout = (uint32_t)min<uint64_t>(pcnt < nbt ? nbt - pcnt : 0, tcnt);
+
+    // Values.
+    const V eb = get_eb<V>(st);
+    const uint64_t lo = chunk_lo(g, t), nt = chunk_len(g, t);
+    if (MODE == 1 && first && tid == 0) out[lo] = (V)(int32_t)head * eb;
+    // Values of the chunk's last block (mode 2: of its last unit's block).
+    const uint32_t Llast =
+        nbt ? (uint32_t)(nt - 1 - (nbt - 1) * (uint64_t)B) : 0u;
+    const uint32_t Lfull = MODE == 2 ? B - 1 : B;
+    uint32_t segbase = carry;
+    for (uint32_t base = 0; base < nout; base += kFusedSeg) {
+        if (tcnt > kFusedSeg) {
+            __syncthreads();
+            fill_list(base);
+            __syncthreads();
+            if (MODE == 1) {
+                const uint32_t ws = seg_sum(min(tcnt - base, kFusedSeg));
+                if (lane == 0) s_sum[wv] = ws;
+                __syncthreads();
+            }
+        }
+        uint32_t wbase = segbase;
+        if (MODE == 1) {
+#pragma unroll
+            for (uint32_t w = 0; w < kWG / 64; ++w) {
+                const uint32_t v = uniform(s_sum[w]);
+                wbase += w < wv ? v : 0u;
+                segbase += v;
+            }
+        }
+        uint32_t a, z;
+        const uint32_t nseg = min(tcnt - base, kFusedSeg);
+        wave_steps(nseg, a, z);
+        uint32_t e = list[min(a * KS + ld, nseg - 1)];
+        for (uint32_t q = a; q < z; ++q) {
+            const uint32_t j = q * KS + ld;
+            const bool act = ld < KS && base + j < nout;
+            const uint64_t bi = (uint64_t)pcnt + base + q * KS;  // the step's first block
+            if (bi >= nbt) break;
+            const bool full = FULL8 && (bi + KS < nbt || Llast == Lfull);  // uniform: no short block here
+            uint32_t dl[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+            uint32_t L = Lfull, hq = 0;
+            const uint32_t lp = e & 0xFFFFu, e0 = e;
+            e = list[min(j + KS, nseg - 1)];  // the next step's entry
+            if (act) {
+                if (bi + ld == nbt - 1) L = Llast;
+                if (MODE == 2) __builtin_memcpy(&hq, tb + lp, 4);
+                uint32_t h;
+                if (full) {
+                    bad = bad || e0 >> 31;
+                    decode_octet8<false>(tb, MODE == 2 ? lp + 4 : lp, (e0 >> 16) & 63u, spb, Lfull, lo_, dl);
+                } else
+                    decode_slot(L, false, lo_, tb, MODE == 2 ? lp + 4 : lp, lend, dl, h, bad);
+                if (bi + ld == nbt - 1 && lo_ == 0) {
+                    // The chunk's last block ends where the chunk does (the
+                    // last chunk: inside the stream).
+                    const uint32_t q0 = MODE == 2 ? lp + 4 : lp;
+                    const uint32_t bw = q0 < lend ? tb[q0] : 255u;
+                    const uint64_t e = s + q0 + block_bytes(bw <= 32 && L ? bw : 0u, L);
+                    if ((bw > 32 && L) || (t + 1 < g.T ? e != ae : e > len)) bad = true;
+                }
+            }
+            const uint32_t v = act ? dl[7] : 0u;
+            const uint32_t incl = wave_incl_scan_u32(v, lane);
+            const uint32_t ex = incl - v;
+            if (MODE == 1) {
+                const uint32_t q0 = wbase + ex;
+                wbase += __builtin_amdgcn_readlane(incl, 63);
+                if (act) {
+                    V *dst = out + lo + 1 + (bi + ld) * B + 8 * lo_;
+                    V y[8];
+#pragma unroll
+                    for (int k = 0; k < 8; ++k) y[k] = (V)(int32_t)(q0 + dl[k]) * eb;
+                    if (full) {
+                        store_octet_out<sizeof(V) == 4>(dst, y);
+                    } else {
+#pragma unroll
+                        for (int k = 0; k < 8; ++k)
+                            if (8 * lo_ + k < L) dst[k] = y[k];
+                    }
+                }
+            } else {
+                const uint32_t q0 = hq + ex - (uint32_t)__shfl((int)ex, lane - (int)lo_);
+                if (act) {
+                    V *dst = out + lo + (bi + ld) * B + 8 * lo_;
+                    V y[8];
+                    y[0] = (V)(int32_t)q0 * eb;
+#pragma unroll
+                    for (int k = 1; k < 8; ++k) y[k] = (V)(int32_t)(q0 + dl[k - 1]) * eb;
+                    if (full) {
+                        store_octet_out<sizeof(V) == 4>(dst, y);
+                    } else {
+#pragma unroll
+                        for (int k = 0; k < 8; ++k)
+                            if (8 * lo_ + k <= L) dst[k] = y[k];
+                    }
+                }
+            }
+        }
+    }
+    if (bad) raise_error(ctl, kErrStream);
 }
 
 // ---------------------------------------------------------------------------
@@ -3477,6 +4128,36 @@ uint64_t decompress_ws_layout(const Geom &g, uint64_t len, uint8_t *base, Decomp
     return off;
 }
 
+// Workspace of the fused parse and decode: control block, chunk table, then
+// the words a call clears (per tile an exit, a first word and a current word;
+// per group of tiles a word, kGroupStride apart).
+struct FusedWs {
+    uint32_t *ctl;
+    uint64_t *ctab;
+    uint64_t *exit_st;
+    FusedStatus S;
+    uint64_t nclr;
+};
+
+uint64_t fused_tiles(const Geom &g, const FusedShape &f, uint64_t len) { return len / f.S + 1 + g.T; }
+
+uint64_t fused_ws_layout(const Geom &g, const FusedShape &f, uint64_t len, uint8_t *base, FusedWs *w)
+{
+    const uint64_t nt = fused_tiles(g, f, len);
+    uint64_t off = align_up(64);
+    if (w) w->ctl = reinterpret_cast<uint32_t *>(base);
+    if (w) w->ctab = reinterpret_cast<uint64_t *>(base + off);
+    off += align_up(8 * (3ull * g.T + 1));
+    if (w) {
+        w->exit_st = reinterpret_cast<uint64_t *>(base + off);
+        w->S.own = w->exit_st + nt;
+        w->S.st = w->S.own + nt;
+        w->S.gst = w->S.st + nt;
+        w->nclr = 3 * nt + kGroupStride * lb_groups(nt);
+    }
+    return align_up(off + 8 * (3 * nt + kGroupStride * lb_groups(nt)));
+}
+
 }  // namespace
 
 uint64_t index_bytes(uint64_t n, int B, int T, int mode)
@@ -3505,7 +4186,11 @@ uint64_t decompress_workspace_bytes(uint64_t stream_bytes, uint64_t n, int B, in
 {
     Geom g;
     if (!make_geom(n, B, T, &g, 4, (uint32_t)mode)) return 0;
-    return decompress_ws_layout(g, stream_bytes, nullptr, nullptr);
+    const uint64_t two = decompress_ws_layout(g, stream_bytes, nullptr, nullptr);
+    FusedShape f;
+    return fused_shape(g, stream_bytes, &f)
+               ? std::max(two, fused_ws_layout(g, f, stream_bytes, nullptr, nullptr))
+               : two;
 }
 
 uint32_t *workspace_error_word(void *d_work)
@@ -3779,6 +4464,35 @@ int launch_compress_noalloc(const float *d_x, uint64_t n, int err_mode, double a
 }
 
 template <typename V>
+static int launch_fused(const Geom &g, const FusedShape &f, const FusedWs &w, const uint8_t *d_stream,
+                        uint64_t len, V *d_out, hipStream_t stream)
+{
+    LookbackOrder order(stream);
+    const uint32_t cgrid = (uint32_t)std::min<uint64_t>((w.nclr + kWG - 1) / kWG, 1024);
+    SZP_LAUNCH("k_fused_setup", k_fused_setup, dim3(cgrid), dim3(kWG), 0, stream, d_stream, len, g,
+               f.S, w.ctab, w.exit_st, w.nclr, w.ctl);
+    const dim3 grid((uint32_t)fused_tiles(g, f, len));
+    const uint32_t nbuf = fused_buf_bytes(f), nword = fused_bitmap_words(f);
+    const uint32_t lds = nbuf + 4 * nword + 4 * kFusedSeg;
+#define SZP_FUSED(M, F8)                                                                         \
+    SZP_LAUNCH("k_fused_decode", (k_fused_decode<V, M, F8>), grid, dim3(kWG), lds, stream,       \
+               d_stream, len, g, f, nbuf, nword, w.ctab, w.exit_st, w.S, d_out, w.ctl)
+    if (g.mode == 2) {
+        if (g.B & 7)
+            SZP_FUSED(2, false);
+        else
+            SZP_FUSED(2, true);
+    } else {
+        if (g.B & 7)
+            SZP_FUSED(1, false);
+        else
+            SZP_FUSED(1, true);
+    }
+#undef SZP_FUSED
+    return hipGetLastError() == hipSuccess ? kOk : kHip;
+}
+
+template <typename V>
 static int launch_decompress_t(int mode, const uint8_t *d_stream, uint64_t len, uint64_t n, int B,
                                int T, V *d_out, void *d_work, uint64_t work_bytes,
                                hipStream_t stream)
@@ -3788,6 +4502,13 @@ static int launch_decompress_t(int mode, const uint8_t *d_stream, uint64_t len, 
     if (n && !d_out) return kArg;
     if ((reinterpret_cast<uintptr_t>(d_stream) & 15) || (reinterpret_cast<uintptr_t>(d_work) & 255))
         return kArg;
+    FusedShape f;
+    if (fused_shape(g, len, &f)) {
+        FusedWs w;
+        if (fused_ws_layout(g, f, len, reinterpret_cast<uint8_t *>(d_work), &w) <= work_bytes &&
+            fused_tiles(g, f, len) <= 0x7fffffffu)
+            return launch_fused<V>(g, f, w, d_stream, len, d_out, stream);
+    }
     DecompressWs w;
     if (decompress_ws_layout(g, len, reinterpret_cast<uint8_t *>(d_work), &w) > work_bytes)
         return kCap;
