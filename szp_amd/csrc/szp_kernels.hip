@@ -2154,26 +2154,23 @@ __device__ __forceinline__ void copy_out_nt(uint8_t *__restrict__ dst, uint32_t 
 // run up to 32 bytes past it, inside the buffer's slack).  dl[i] = inclusive
 // prefix of the slot's deltas, or the absolute head value in dl[0] for a head
 // slot (h = 1).  Returns the number of values (0 for idle slots); sets bad on
-// an invalid width or a block that overruns the bytes present.  FULL: the
-// caller guarantees a full octet (8 * o + 8 <= L), so no value is masked.
-template <bool FULL = false>
+// an invalid width or a block that overruns the bytes present.  Full octets of
+// whole blocks take decode_octet8.
 __device__ __forceinline__ uint32_t decode_slot(uint32_t L, bool head, uint32_t o,
                                                 const uint8_t *buf, uint32_t lp, uint32_t lend,
                                                 uint32_t dl[8], uint32_t &h, bool &bad)
 {
     h = 0;
-    if (!FULL) {
 #pragma unroll
-        for (int i = 0; i < 8; ++i) dl[i] = 0;
-        if (head) {
-            if (o) return 0;
-            h = 1;
-            __builtin_memcpy(&dl[0], buf + lp, 4);
-            return 1;
-        }
-        if (8 * o >= L) return 0;
+    for (int i = 0; i < 8; ++i) dl[i] = 0;
+    if (head) {
+        if (o) return 0;
+        h = 1;
+        __builtin_memcpy(&dl[0], buf + lp, 4);
+        return 1;
     }
-    const uint32_t m = FULL ? 8u : min(8u, L - 8 * o);
+    if (8 * o >= L) return 0;
+    const uint32_t m = min(8u, L - 8 * o);
     // A bad width or a block past the bytes present is reported and decoded
     // as width 0; every path below writes all of dl (no early exit, so the
     // compiler need not clear dl at each branch).
@@ -2231,7 +2228,7 @@ __device__ __forceinline__ uint32_t decode_slot(uint32_t L, bool head, uint32_t 
         const uint32_t mag = (v[i] << r) | low;
         // s = ~0 when sign bit 7 - i is set; (mag ^ s) - s is then 0 - mag.
         const uint32_t s = (uint32_t)((int32_t)(sg << (24 + i)) >> 31);
-        if (FULL || (uint32_t)i < m) run += (mag ^ s) - s;
+        if ((uint32_t)i < m) run += (mag ^ s) - s;
         dl[i] = run;
     }
     return m;
@@ -2321,6 +2318,18 @@ __device__ __forceinline__ uint32_t decode_octet8(const uint8_t *buf, uint32_t l
         v[4] = c.x; v[5] = c.y; v[6] = c.z; v[7] = c.w;
     }
     return octet_signed<SUM>(v, r, res, sg, dl);
+}
+
+// decode_octet8 of the block at buf[lp], its width byte read and checked: an
+// invalid width or a block past lend sets bad and is decoded as width 0.
+__device__ __forceinline__ void decode_block8(const uint8_t *buf, uint32_t lp, uint32_t spb, uint32_t o,
+                                              uint32_t lend, uint32_t dl[8], bool &bad)
+{
+    const uint32_t b = buf[lp];
+    const uint32_t n = b ? __umul24(spb, b + 1) + 1 : 1u;  // block_bytes(b, 8 * spb)
+    const bool ok = b <= 32 && lp + n <= lend;
+    if (!ok) bad = true;
+    decode_octet8<false>(buf, lp, ok ? b : 0u, spb, 8 * spb, o, dl);
 }
 
 // Segmented scan of slot aggregates (h, v) in slot order: a head restarts
@@ -2441,12 +2450,10 @@ __device__ __forceinline__ bool decode_simple_fast(
 #pragma unroll
         for (int r = 0; r < kMaxRounds; ++r) {
             if ((uint32_t)r * K < nti) {
-                uint32_t h;
                 if (pos[r] < P0 || pos[r] >= P1)
                     bad = true;
                 else
-                    decode_slot<true>(B, false, o, buf, (uint32_t)(pos[r] - tbase), lend, dl[r], h,
-                                      bad);
+                    decode_block8(buf, (uint32_t)(pos[r] - tbase), SPB, o, lend, dl[r], bad);
             }
         }
     } else if (!bad) {
@@ -2466,12 +2473,11 @@ __device__ __forceinline__ bool decode_simple_fast(
             if (!ok) {
                 bad = true;
             } else if ((uint32_t)r * K < nti) {
-                uint32_t h;
                 if (pos[r] < Pr || pos[r] >= Pn)
                     bad = true;
                 else
-                    decode_slot<true>(B, false, o, buf, (uint32_t)(pos[r] - rbase), (uint32_t)(Pn - rbase),
-                                dl[r], h, bad);
+                    decode_block8(buf, (uint32_t)(pos[r] - rbase), SPB, o, (uint32_t)(Pn - rbase), dl[r],
+                                  bad);
             }
         }
     }
@@ -3534,7 +3540,7 @@ __device__ __forceinline__ void pipe_decode(const PipeTile &p, uint32_t carry, V
                                             V *__restrict__ out, uint32_t *__restrict__ ctl,
                                             DecodeLds &L)
 {
-    constexpr uint32_t K = 256 / SPB, B = 8 * SPB;
+    constexpr uint32_t K = 256 / SPB;
     const int tid = threadIdx.x, lane = __lane_id(), wv = tid >> 6;
     const uint32_t d = (uint32_t)tid / SPB, o = (uint32_t)tid % SPB;
     const uint32_t lend = (uint32_t)(p.P1 - (p.P0 & ~15ull));
@@ -3547,8 +3553,7 @@ __device__ __forceinline__ void pipe_decode(const PipeTile &p, uint32_t carry, V
     for (int r = 0; r < kMaxRounds; ++r) {
         const uint32_t lp0 = L.s_pos[r * K + d];
         if (lp0 == ~0u) bad = true;
-        uint32_t h;
-        decode_slot<true>(B, false, o, L.buf, lp0 == ~0u ? 0u : lp0, lend, dl[r], h, bad);
+        decode_block8(L.buf, lp0 == ~0u ? 0u : lp0, SPB, o, lend, dl[r], bad);
     }
     if (bad) raise_error(ctl, kErrStream);
     uint32_t ex[kMaxRounds];
@@ -3970,7 +3975,7 @@ __global__ __launch_bounds__(kWG, 7) void k_batch_compress_once(const BatchJob *
                                             J.d_size, J.idx_pos, J.idx_carry, e.tile, L);
 }
 
-template <int SPB>
+// Block sizes without a fast path (B / 8 not a power of two up to 32).
 __global__ __launch_bounds__(kWG) void k_batch_decode(const BatchJob *__restrict__ jobs,
                                                       const QEntry *__restrict__ qmap,
                                                       uint64_t total, uint64_t *queue,
@@ -3991,10 +3996,139 @@ __global__ __launch_bounds__(kWG) void k_batch_decode(const BatchJob *__restrict
             const QEntry e = qmap[q];
             const BatchJob &J = jobs[e.job];
             const Geom g = J.g;
-            decode_tile<float, true, SPB>(J.st, J.cap, g, J.idx_pos, J.idx_carry, J.y, nullptr,
+            decode_tile<float, true, 0>(J.st, J.cap, g, J.idx_pos, J.idx_carry, J.y, nullptr,
                                           ctl, e.tile, L);
             __syncthreads();
         }
+    }
+}
+
+// The pipelined decode (k_decode_pipe) over the batch's queue: while a tile is
+// unpacked, the next one's stream bytes, positions and carry are in flight, and
+// the queue entry of the one after it is fetched.  Entries are handed out by
+// class as there (class c of C: entries c, c + C, ...; ctr = its counters, 8
+// words apart), `ticket` consecutive ones of the class at a time, the first
+// two tickets of a workgroup fixed.  Tiles that do not go through the pipeline
+// (chunk heads, short blocks, a field's last tile, short chunks, over
+// kPipeBytes) are decoded in their turn by decode_tile; its loads wait for the
+// next tile's, which a workgroup's neighbours cover.  A malformed stream raises
+// the error word; the other tiles are decoded all the same.
+// 256 fields of 64 KB to 64 MB (2.35 GB, REL 1e-3, B = 128): 864 us one tile
+// after another (loads, unpacking and a read of the error word in turn) ->
+// 724 us; 713-756 us over tickets of 1 to 8 and grids of 1 to 2 residencies.
+struct BatchTile {
+    PipeTile p;
+    uint32_t job;
+    float eb;
+};
+
+__device__ __forceinline__ BatchTile batch_plan(const BatchJob *__restrict__ jobs, QEntry e, bool any)
+{
+    BatchTile t;
+    t.job = any ? e.job : 0u;
+    const BatchJob &J = jobs[t.job];
+    t.p = pipe_plan(J.st, J.g, J.idx_pos, any ? e.tile : ~0ull);
+    if (J.g.R != (uint32_t)kMaxRounds) t.p.simple = false;
+    t.eb = get_eb<float>(J.st);
+    return t;
+}
+
+template <int SPB>
+__global__ __launch_bounds__(kWG, 4) void k_batch_decode_pipe(const BatchJob *__restrict__ jobs,
+                                                           const QEntry *__restrict__ qmap,
+                                                           uint64_t total, uint32_t *ctr,
+                                                           uint32_t ticket, uint32_t *ctl)
+{
+    __shared__ DecodeLds L;
+    __shared__ uint32_t s_ent[3];  // the entry after next: job, tile, 1 when there is one
+    const uint32_t tid = threadIdx.x;
+    const uint32_t G = gridDim.x, C = min(G, kPipeClasses);
+    const uint32_t c = blockIdx.x % C, r = blockIdx.x / C, nper = (G - c + C - 1) / C;
+    const uint32_t cn = c < total ? (uint32_t)((total - c + C - 1) / C) : 0u;  // the class's entries
+    ctr += 8 * c;
+    // Entry k of this workgroup is the class's entry k % ticket of ticket
+    // k / ticket: r, r + nper, then the counter's.
+    auto clip = [](uint64_t i) { return (uint32_t)min<uint64_t>(i, 0xFFFFFFFFu); };  // none: >= cn
+    const uint32_t cur_i = clip((uint64_t)r * ticket);
+    uint32_t nxt_i = ticket > 1 ? clip((uint64_t)r * ticket + 1) : r + nper;
+    uint32_t sub = ticket > 1 ? 1u : 0u;     // of the next entry, in its ticket
+    uint32_t fixed = ticket > 1 ? 1u : 0u;   // fixed tickets not yet begun
+    QEntry e = qmap[min(c + (uint64_t)C * cur_i, total - 1)];
+    BatchTile cur = batch_plan(jobs, e, cur_i < cn);
+    uint4 rb[kPipeVec];
+    uint64_t pos[kMaxRounds];
+    uint32_t carry = 0;
+    bool have = pipe_issue<SPB>(jobs[cur.job].st, jobs[cur.job].cap, jobs[cur.job].idx_pos,
+                                jobs[cur.job].idx_carry, cur.p, rb, pos, carry);
+    e = qmap[min(c + (uint64_t)C * nxt_i, total - 1)];
+    bool any = nxt_i < cn;
+    while (cur.p.tile != ~0ull) {
+        constexpr uint32_t K = 256 / SPB;
+        const uint32_t d = tid / SPB, o = tid % SPB;
+        const BatchTile nxt = batch_plan(jobs, e, any);
+        const uint32_t ccur = carry;
+        if (have) {
+            const uint64_t a0 = cur.p.P0 & ~15ull;
+#pragma unroll
+            for (int v = 0; v < kPipeVec; ++v) {
+                const uint32_t q = 16u * (tid + (uint32_t)kWG * v);
+                if (a0 + q < cur.p.P1) *reinterpret_cast<uint4 *>(L.buf + q) = rb[v];
+            }
+            if (o == 0) {
+#pragma unroll
+                for (int q = 0; q < kMaxRounds; ++q)
+                    L.s_pos[q * K + d] = (pos[q] >= cur.p.P0 && pos[q] < cur.p.P1)
+                                             ? (uint32_t)(pos[q] - a0)
+                                             : ~0u;
+            }
+        }
+        // The entry after next: the rest of the ticket, the second fixed
+        // ticket or a new one (asked for now, used after the next tile's loads
+        // are out; see k_decode_pipe for the register zero).
+        uint32_t got = 0;
+        const bool go_on = sub + 1 < ticket;
+        const bool ask = any && !go_on && !fixed;
+        if (tid == 0 && ask) {
+            uint32_t z;
+            asm volatile("v_mov_b32 %0, 0" : "=v"(z));
+            got = atomicAdd(ctr + z, 1u);
+        }
+        __syncthreads();
+        const bool have_n = pipe_issue<SPB>(jobs[nxt.job].st, jobs[nxt.job].cap, jobs[nxt.job].idx_pos,
+                                            jobs[nxt.job].idx_carry, nxt.p, rb, pos, carry);
+        QEntry en{0, 0};
+        uint32_t ni = 0;
+        if (tid == 0) {
+            ni = go_on ? nxt_i + 1
+                       : clip((fixed ? (uint64_t)r + nper : 2ull * nper + got) * (uint64_t)ticket);
+            en = qmap[min(c + (uint64_t)C * ni, total - 1)];
+        }
+        if (have) {
+            pipe_decode<float, SPB>(cur.p, ccur, cur.eb, jobs[cur.job].y, ctl, L);
+        } else {
+            const BatchJob &J = jobs[cur.job];
+            const Geom g = J.g;
+            decode_tile<float, true, SPB>(J.st, J.cap, g, J.idx_pos, J.idx_carry, J.y, nullptr, ctl,
+                                          cur.p.tile, L);
+        }
+        if (tid == 0) {
+            s_ent[0] = en.job;
+            s_ent[1] = en.tile;
+            s_ent[2] = any ? ni : ~0u;
+        }
+        __syncthreads();  // L and s_ent are reused by the next step
+        if (go_on) {
+            ++sub;
+        } else {
+            sub = 0;
+            fixed = 0;
+        }
+        have = have_n;
+        cur = nxt;
+        e.job = uniform(s_ent[0]);
+        e.tile = uniform(s_ent[1]);
+        nxt_i = uniform(s_ent[2]);
+        any = nxt_i < cn;
     }
 }
 
@@ -4818,19 +4952,26 @@ int batch_launch(const BatchPlan &P, uint32_t ticket, uint32_t grid, hipStream_t
     uint64_t *status = reinterpret_cast<uint64_t *>(base + P.status);
     BatchJob *jobs = reinterpret_cast<BatchJob *>(base + P.jobs);
     const QEntry *qmap = reinterpret_cast<const QEntry *>(base + P.qmap);
-    const uint32_t cgrid = (uint32_t)std::min<uint64_t>((P.nstatus + kWG - 1) / kWG, 4096);
-    SZP_LAUNCH("k_clear", k_clear, dim3(cgrid), dim3(kWG), 0, stream, ctl, status, P.nstatus);
+    // Decompress: the 256 bytes of ticket counters (batch_layout rounds the
+    // one status word up to them).
+    const uint64_t nclr = P.decode ? std::max<uint64_t>(P.nstatus, 32) : P.nstatus;
+    const uint32_t cgrid = (uint32_t)std::min<uint64_t>((nclr + kWG - 1) / kWG, 4096);
+    SZP_LAUNCH("k_clear", k_clear, dim3(cgrid), dim3(kWG), 0, stream, ctl, status, nclr);
     const dim3 block(kWG);
     if (P.decode) {
+        if (P.spb == 0) {
+            const uint32_t gr = grid ? grid : resident_grid(k_batch_decode);
+            SZP_LAUNCH("k_batch_decode", k_batch_decode, dim3(gr), block, 0, stream, jobs, qmap,
+                       P.tiles, status, ticket, ctl);
+        }
         switch (P.spb) {
 #define SZP_BATCH_DECODE_CASE(S)                                                                 \
     case S: {                                                                                    \
-        const uint32_t gr = grid ? grid : resident_grid(k_batch_decode<S>);                      \
-        SZP_LAUNCH("k_batch_decode", k_batch_decode<S>, dim3(gr), block, 0, stream, jobs, qmap,  \
-                   P.tiles, status, ticket, ctl);                                                \
+        const uint32_t gr = grid ? grid : resident_grid(k_batch_decode_pipe<S>);                 \
+        SZP_LAUNCH("k_batch_decode", k_batch_decode_pipe<S>, dim3(gr), block, 0, stream, jobs,   \
+                   qmap, P.tiles, reinterpret_cast<uint32_t *>(status), ticket, ctl);            \
         break;                                                                                   \
     }
-            SZP_BATCH_DECODE_CASE(0)
             SZP_BATCH_DECODE_CASE(1)
             SZP_BATCH_DECODE_CASE(2)
             SZP_BATCH_DECODE_CASE(4)
@@ -4889,7 +5030,7 @@ uint32_t batch_resident_grid(const BatchPlan &P)
 {
     // Occupancy does not depend on the template arguments' SPB beyond
     // registers, which the SPB = 16 forms bound.
-    if (P.decode) return resident_grid(k_batch_decode<16>);
+    if (P.decode) return resident_grid(k_batch_decode_pipe<16>);
     return P.index ? resident_grid(k_batch_compress<true, 16>) : resident_grid(k_batch_compress<false, 16>);
 }
 
