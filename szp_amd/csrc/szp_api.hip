@@ -12,8 +12,12 @@
 #include <string.h>
 
 #include <algorithm>
+#include <atomic>
 #include <mutex>
 #include <string>
+#include <system_error>
+#include <thread>
+#include <vector>
 
 #include "szp.h"
 #include "szp_amd.h"
@@ -52,9 +56,124 @@ int map_device_errors(uint32_t bits)
     return SZP_AMD_OK;
 }
 
+// Copies between host arrays and device buffers go through pinned staging
+// buffers, filled and emptied by several threads: one thread copies memory at
+// less than the link's rate, and the runtime's own pageable copies reach 25
+// GB/s to the device and 18 from it, against 55 and 57 from pinned memory.
+// 2^24 floats compressed and decompressed (sinusoids, ABS 1e-3): 7.0 -> 3.5 ms;
+// below kCopyStaged the threads cost as much as they save (2^21 floats: 1.00 ->
+// 0.81 ms, 2^16: no change).
+constexpr int kCopyThreads = 4;             // at most; each owns kCopySlots buffers
+constexpr int kCopySlots = 2;               // one in flight while the other is filled or emptied
+constexpr size_t kCopyChunk = 2u << 20;     // bytes of a buffer
+constexpr size_t kCopyStaged = 8u << 20;    // smaller copies are left to the runtime
+
+int copy_threads()
+{
+    cpu_set_t set;
+    const int cpus = sched_getaffinity(0, sizeof(set), &set) == 0 ? CPU_COUNT(&set) : 1;
+    return std::min(cpus, kCopyThreads);
+}
+
+// Pinned buffers of one device's session, with a stream and events for each
+// copying thread.  Held with the session's device buffers (16 MiB).
+struct Staging {
+    struct Lane {
+        hipStream_t stream = nullptr;
+        unsigned char *buf[kCopySlots] = {};
+        hipEvent_t ev[kCopySlots] = {};
+    };
+    Lane lane[kCopyThreads];
+    bool ready = false;
+
+    bool ensure()
+    {
+        if (ready) return true;
+        for (Lane &l : lane) {
+            if (!l.stream && hipStreamCreateWithFlags(&l.stream, hipStreamNonBlocking) != hipSuccess)
+                return false;
+            for (int k = 0; k < kCopySlots; ++k) {
+                if (!l.buf[k] && hipHostMalloc((void **)&l.buf[k], kCopyChunk, 0) != hipSuccess) {
+                    l.buf[k] = nullptr;
+                    return false;
+                }
+                if (!l.ev[k] && hipEventCreateWithFlags(&l.ev[k], hipEventDisableTiming) != hipSuccess) {
+                    l.ev[k] = nullptr;
+                    return false;
+                }
+            }
+        }
+        return ready = true;
+    }
+
+    // Copies n bytes between host memory and the device; work enqueued on
+    // `stream` afterwards sees a copy to the device, and a copy to the host is
+    // complete on return.
+    bool copy(void *dst, const void *src, size_t n, bool to_device, hipStream_t stream)
+    {
+        const int nt = copy_threads();
+        if (n < kCopyStaged || nt < 2 || !ensure()) {
+            if (to_device)
+                return hipMemcpyAsync(dst, src, n, hipMemcpyHostToDevice, stream) == hipSuccess;
+            return hipMemcpy(dst, src, n, hipMemcpyDeviceToHost) == hipSuccess;
+        }
+        int dev = 0;
+        if (hipGetDevice(&dev) != hipSuccess) return false;
+        std::atomic<bool> ok{true};
+        std::atomic<size_t> next{0};
+        const size_t chunks = (n + kCopyChunk - 1) / kCopyChunk;
+        auto size_of = [&](size_t c) { return std::min(kCopyChunk, n - c * kCopyChunk); };
+        auto work = [&](int w) {
+            Lane &l = lane[w];
+            bool good = hipSetDevice(dev) == hipSuccess;
+            size_t held[kCopySlots];  // the chunk a slot holds, when busy
+            bool busy[kCopySlots] = {};
+            auto settle = [&](int k) {
+                if (!busy[k]) return;
+                busy[k] = false;
+                good = hipEventSynchronize(l.ev[k]) == hipSuccess && good;
+                if (!to_device && good)
+                    memcpy((unsigned char *)dst + held[k] * kCopyChunk, l.buf[k], size_of(held[k]));
+            };
+            int k = 0;
+            for (size_t c; good && (c = next.fetch_add(1)) < chunks; k = (k + 1) % kCopySlots) {
+                settle(k);
+                const size_t at = c * kCopyChunk, m = size_of(c);
+                if (to_device) {
+                    memcpy(l.buf[k], (const unsigned char *)src + at, m);
+                    good = good && hipMemcpyAsync((unsigned char *)dst + at, l.buf[k], m,
+                                                  hipMemcpyHostToDevice, l.stream) == hipSuccess;
+                } else {
+                    good = good && hipMemcpyAsync(l.buf[k], (const unsigned char *)src + at, m,
+                                                  hipMemcpyDeviceToHost, l.stream) == hipSuccess;
+                }
+                good = good && hipEventRecord(l.ev[k], l.stream) == hipSuccess;
+                held[k] = c;
+                busy[k] = good;
+            }
+            for (int j = 0; j < kCopySlots; ++j) settle((k + j) % kCopySlots);
+            // Nothing may still use the buffers after an error.
+            if (!good) (void)hipStreamSynchronize(l.stream);
+            if (!good) ok = false;
+        };
+        std::vector<std::thread> th;
+        const int want = (int)std::min<size_t>(nt, chunks);
+        try {
+            th.reserve((size_t)want);
+            for (int w = 1; w < want; ++w) th.emplace_back(work, w);
+        } catch (const std::exception &) {
+            // No thread to be had: those that run share the chunks.
+        }
+        work(0);
+        for (auto &t : th) t.join();
+        return ok;
+    }
+};
+
 // Device buffers reused by the host-pointer entry points of one device.
 struct Session {
     std::mutex mu;
+    Staging staging;
     hipStream_t stream = nullptr;
     void *buf[4] = {nullptr, nullptr, nullptr, nullptr};
     size_t cap[4] = {0, 0, 0, 0};
@@ -187,8 +306,7 @@ int host_compress(int fast, int dtype, const void *data, uint64_t n, int mode, d
     void *d_ws = s->ensure(2, wsb);
     uint64_t *d_size = (uint64_t *)s->ensure(3, 256);
     if (!d_in || !d_out || !d_ws || !d_size) return SZP_AMD_ERR_NOMEM;
-    if (n && hipMemcpyAsync(d_in, data, n * vb, hipMemcpyHostToDevice, s->stream) != hipSuccess)
-        return SZP_AMD_ERR_HIP;
+    if (n && !s->staging.copy(d_in, data, n * vb, true, s->stream)) return SZP_AMD_ERR_HIP;
     int rc = launch_compress(dtype, d_in, n, mode, abs_eb, rel, B, T, d_out, cap, d_size, d_ws,
                              wsb, s->stream, nullptr, 0, fast);
     if (rc) return rc;
@@ -198,7 +316,7 @@ int host_compress(int fast, int dtype, const void *data, uint64_t n, int mode, d
     if (hipMemcpy(&size, d_size, 8, hipMemcpyDeviceToHost) != hipSuccess) return SZP_AMD_ERR_HIP;
     unsigned char *dst = into ? into : (unsigned char *)malloc(size ? size : 1);
     if (!dst) return SZP_AMD_ERR_NOMEM;
-    if (hipMemcpy(dst, d_out, size, hipMemcpyDeviceToHost) != hipSuccess) {
+    if (!s->staging.copy(dst, d_out, size, false, s->stream)) {
         if (!into) free(dst);
         return SZP_AMD_ERR_HIP;
     }
@@ -227,7 +345,7 @@ int host_decompress(int fast, int dtype, const unsigned char *eb_be, const unsig
     void *d_ws = s->ensure(2, wsb);
     if (!d_st || !d_out || !d_ws) return SZP_AMD_ERR_NOMEM;
     if (hipMemcpyAsync(d_st, eb_be, vb, hipMemcpyHostToDevice, s->stream) != hipSuccess ||
-        hipMemcpyAsync(d_st + vb, body, blen, hipMemcpyHostToDevice, s->stream) != hipSuccess)
+        !s->staging.copy(d_st + vb, body, blen, true, s->stream))
         return SZP_AMD_ERR_HIP;
     int rc = launch_decompress(dtype, d_st, len, n, B, T, d_out, d_ws, wsb, s->stream, fast);
     if (rc) return rc;
@@ -235,7 +353,7 @@ int host_decompress(int fast, int dtype, const unsigned char *eb_be, const unsig
     if (rc) return rc;
     void *dst = into ? into : malloc(n ? n * vb : vb);
     if (!dst) return SZP_AMD_ERR_NOMEM;
-    if (n && hipMemcpy(dst, d_out, n * vb, hipMemcpyDeviceToHost) != hipSuccess) {
+    if (n && !s->staging.copy(dst, d_out, n * vb, false, s->stream)) {
         if (!into) free(dst);
         return SZP_AMD_ERR_HIP;
     }
