@@ -2117,6 +2117,51 @@ __device__ __forceinline__ void store_octet_out(V *p, const V y[8])
     }
 }
 
+// Writes a wave's 512 values, lane l holding wp[8 l .. 8 l + 7], every lane
+// active.  NT: non-temporal (float only).
+//
+// Double: the lanes of a quad exchange their 16-byte pieces over DPP, so that
+// each of the four store instructions writes 64-byte runs; a lane's own pieces
+// in turn would be 16-byte runs 64 bytes apart, four times the requests to the
+// L2 (384^3 field: foreign-stream decode 212 -> 159 us, pipelined decode 159 ->
+// 141 us; non-temporal 463 and 489 us).  Float octets are two pieces, 32 bytes
+// apart, and gain nothing from the exchange (335 us either way on the 512^3
+// field, the pipelined decode 147 -> 149 us).
+template <bool NT>
+__device__ __forceinline__ void store_wave(float *wp, const float y[8])
+{
+    store_octet_out<NT>(wp + 8 * __lane_id(), y);
+}
+// Row K of the quad's four: lane i writes piece i of lane K's values u.
+template <int K>
+__device__ __forceinline__ void store_quad_row(double *p, const uint32_t u[16], uint32_t i)
+{
+    typedef uint32_t u4 __attribute__((ext_vector_type(4), aligned(4)));
+    u4 w;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+        auto of = [&](uint32_t v) {  // v of lane K of the quad
+            return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, K * 0x55, 0xF, 0xF, true);
+        };
+        const uint32_t a = of(u[k]), b = of(u[4 + k]), c = of(u[8 + k]), d = of(u[12 + k]);
+        const uint32_t lo = i & 1 ? b : a, hi = i & 1 ? d : c;
+        w[k] = i & 2 ? hi : lo;
+    }
+    *reinterpret_cast<u4 *>(p + 8 * K) = w;
+}
+template <bool NT>
+__device__ __forceinline__ void store_wave(double *wp, const double y[8])
+{
+    const uint32_t l = __lane_id(), i = l & 3;
+    uint32_t u[16];
+    __builtin_memcpy(u, y, 64);
+    double *p = wp + 32 * (l >> 2) + 2 * i;
+    store_quad_row<0>(p, u, i);
+    store_quad_row<1>(p, u, i);
+    store_quad_row<2>(p, u, i);
+    store_quad_row<3>(p, u, i);
+}
+
 // Writes tot bytes (a multiple of 4) from LDS src to dst[0, tot) with
 // non-temporal stores: 16-byte stores for the aligned middle, each store
 // instruction of a wave covering 1 KiB of whole lines, and 4-byte stores for
@@ -2555,7 +2600,7 @@ __device__ __forceinline__ bool decode_simple_fast(
             V y[8];
 #pragma unroll
             for (int i = 0; i < 8; ++i) y[i] = (V)(int32_t)(q0 + dl[r][i]) * eb;
-            store_octet_out<false>(out + Et + (uint64_t)r * 2048u + 8u * (uint32_t)tid, y);
+            store_wave<false>(out + Et + (uint64_t)r * 2048u + 512u * uniform((uint32_t)wv), y);
         }
     }
     return true;
@@ -2637,7 +2682,11 @@ __device__ __forceinline__ bool decode_units_fast(
             y[0] = (V)(int32_t)q0 * eb;
 #pragma unroll
             for (int i = 1; i < 8; ++i) y[i] = (V)(int32_t)(q0 + dl[r][i - 1]) * eb;
-            store_octet_out<sizeof(V) == 4>(out + Et + (uint64_t)r * 2048u + 8u * (uint32_t)tid, y);
+            V *wp = out + Et + (uint64_t)r * 2048u + 512u * uniform((uint32_t)tid >> 6);
+            if (__ballot(true) == ~0ull)
+                store_wave<true>(wp, y);
+            else
+                store_octet_out<sizeof(V) == 4>(wp + 8 * lane, y);
         }
     }
     return true;
@@ -3371,6 +3420,8 @@ __global__ __launch_bounds__(kWG, sizeof(V) == 4 ? 7 : 5) void k_fused_decode(
             const uint64_t bi = (uint64_t)pcnt + base + q * KS;  // the step's first block
             if (bi >= nbt) break;
             const bool full = FULL8 && (bi + KS < nbt || Llast == Lfull);  // uniform: no short block here
+            // Uniform: every lane holds eight values of one run of 512.
+            const bool whole = full && KS * spb == 64 && base + (q + 1) * KS <= nout;
             uint32_t dl[8] = {0, 0, 0, 0, 0, 0, 0, 0};
             uint32_t L = Lfull, hq = 0;
             const uint32_t lp = e & 0xFFFFu, e0 = e;
@@ -3404,7 +3455,9 @@ __global__ __launch_bounds__(kWG, sizeof(V) == 4 ? 7 : 5) void k_fused_decode(
                     V y[8];
 #pragma unroll
                     for (int k = 0; k < 8; ++k) y[k] = (V)(int32_t)(q0 + dl[k]) * eb;
-                    if (full) {
+                    if (whole) {
+                        store_wave<true>(out + lo + 1 + bi * B, y);
+                    } else if (full) {
                         store_octet_out<sizeof(V) == 4>(dst, y);
                     } else {
 #pragma unroll
@@ -3420,7 +3473,9 @@ __global__ __launch_bounds__(kWG, sizeof(V) == 4 ? 7 : 5) void k_fused_decode(
                     y[0] = (V)(int32_t)q0 * eb;
 #pragma unroll
                     for (int k = 1; k < 8; ++k) y[k] = (V)(int32_t)(q0 + dl[k - 1]) * eb;
-                    if (full) {
+                    if (whole) {
+                        store_wave<true>(out + lo + bi * B, y);
+                    } else if (full) {
                         store_octet_out<sizeof(V) == 4>(dst, y);
                     } else {
 #pragma unroll
@@ -3578,7 +3633,7 @@ __device__ __forceinline__ void pipe_decode(const PipeTile &p, uint32_t carry, V
         V y[8];
 #pragma unroll
         for (int i = 0; i < 8; ++i) y[i] = (V)(int32_t)(q0 + dl[r][i]) * eb;
-        store_octet_out<false>(out + p.Et + (uint64_t)r * 2048u + 8u * (uint32_t)tid, y);
+        store_wave<false>(out + p.Et + (uint64_t)r * 2048u + 512u * uniform((uint32_t)wv), y);
     }
 }
 
