@@ -88,7 +88,15 @@ struct Staging {
 
     bool ensure()
     {
-        if (ready) return true;
+        if (!ready) ready = create();
+        // A launch that follows must not find the error of a failed
+        // allocation: the copy then goes the runtime's way.
+        if (!ready) (void)hipGetLastError();
+        return ready;
+    }
+
+    bool create()
+    {
         for (Lane &l : lane) {
             if (!l.stream && hipStreamCreateWithFlags(&l.stream, hipStreamNonBlocking) != hipSuccess)
                 return false;
@@ -103,7 +111,7 @@ struct Staging {
                 }
             }
         }
-        return ready = true;
+        return true;
     }
 
     // Copies n bytes between host memory and the device; work enqueued on

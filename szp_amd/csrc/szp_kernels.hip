@@ -13,10 +13,13 @@
 // and SZp blocks) in element order, a workgroup encodes K items with one
 // thread per 8 elements, and a decoupled look-back over tile byte counts
 // places every tile's output without a second pass over the input.  Decoding
-// recovers block boundaries (the stream has no index) with a speculative
-// parse whose tiles only wait for their predecessor when they cannot
-// synchronise by themselves, then decodes tiles of K blocks with a segmented
-// look-back scan of the Lorenzo deltas.
+// recovers block boundaries (the stream has no index) from byte tiles held in
+// LDS: chains of candidate blocks that meet give a tile its boundary, so tiles
+// only wait for their predecessor when theirs do not, and one look-back gives
+// a tile its first block's number and value; its values are written by the
+// same kernel (B from 8 to 256; other block sizes are parsed by one kernel
+// and decoded by another).  With the side index a persistent kernel decodes
+// tiles of K blocks with no look-back.
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 #include <math.h>
@@ -3874,7 +3877,8 @@ void collect_locked()
 }  // namespace prof
 
 // ---------------------------------------------------------------------------
-// Batched forms: the fields of a batch share one persistent launch.  The
+// Batched forms: the fields of a batch share one launch (decompress with whole
+// blocks: k_batch_decode_pipe, whose queue is shared out over the XCDs).  The
 // host lists every tile of every field in a queue (field by field; a field's
 // tiles in ascending order for compress) and workgroups take `ticket`
 // consecutive queue entries at a time from one atomic counter, running them
@@ -4691,16 +4695,16 @@ static int launch_decompress_t(int mode, const uint8_t *d_stream, uint64_t len, 
     if (n && !d_out) return kArg;
     if ((reinterpret_cast<uintptr_t>(d_stream) & 15) || (reinterpret_cast<uintptr_t>(d_work) & 255))
         return kArg;
-    FusedShape f;
-    if (fused_shape(g, len, &f)) {
-        FusedWs w;
-        if (fused_ws_layout(g, f, len, reinterpret_cast<uint8_t *>(d_work), &w) <= work_bytes &&
-            fused_tiles(g, f, len) <= 0x7fffffffu)
-            return launch_fused<V>(g, f, w, d_stream, len, d_out, stream);
-    }
     DecompressWs w;
     if (decompress_ws_layout(g, len, reinterpret_cast<uint8_t *>(d_work), &w) > work_bytes)
         return kCap;
+    FusedShape f;
+    if (fused_shape(g, len, &f)) {
+        FusedWs fw;
+        if (fused_ws_layout(g, f, len, reinterpret_cast<uint8_t *>(d_work), &fw) <= work_bytes &&
+            fused_tiles(g, f, len) <= 0x7fffffffu)
+            return launch_fused<V>(g, f, fw, d_stream, len, d_out, stream);
+    }
     if (mode == 2 && B == 1) {
         // Units of one value decode as the reference does (k_decode_ra_unit1).
         if (len < g.body) return kArg;

@@ -77,3 +77,18 @@ def test_fused_boundaries(fused_check, fast):
         entries.append((s4, n, B, T, fast))
     out = parse._run(fused_check, entries)
     assert int(out.split("(")[1].split()[0]) > 40, out  # damaged streams among them
+
+
+@pytest.mark.parametrize("n,B,stream", [(1 << 20, 128, 1 << 21), (1 << 20, 8, 1 << 21),
+                                        (1 << 20, 256, 3 << 20), (100003, 32, 200000)])
+def test_short_workspace_is_refused(n, B, stream):
+    """A workspace that holds the block positions of the two-kernel path no
+    more is refused before any launch, also where the fused words would fit:
+    the addresses below are never used.  Those positions alone are 8 bytes a
+    block."""
+    import torch  # noqa: F401  (its HIP runtime is loaded first)
+    import szp_amd as szp
+    short = 8 * (n // B) // 256 * 256
+    rc = szp.lib.szp_amd_decompress_dev(0x10000, stream, n, B, 4, 0x20000, 0x30000, short, None)
+    assert rc == 2  # SZP_AMD_ERR_CAPACITY
+    assert szp.lib.szp_amd_decompress_workspace_size(stream, n, B, 4) > short
