@@ -582,14 +582,16 @@ constexpr uint32_t kFusedNone = 0xFFFFFFFFu;
 // tile's bytes: 14 KiB (seven workgroups' LDS per CU at B = 128), halved while
 // the stream has fewer than 512 tiles (small streams: all CUs work, and the
 // serial walks are short), while floats have fewer than 1024 of more than 8 Ki
-// values, or while a tile would hold more than 64 Ki values (sparse streams:
+// values, or while a tile would hold more than 256 KiB of values (sparse streams:
 // one workgroup writes a tile's values), but at least V.  A tile's boundaries
 // cost the same however long it is, so tiles are halved only for want of work:
 // 2^22 floats REL 1e-4 B=64 with at least 2048 / 1024 / 512 / 256 tiles 54.4 /
 // 36.3 / 34.7 / 34.7 us, 2^22 doubles 67.4 / 50.2 / 37.8 / 38.1, 2^24 doubles
 // REL 1e-2 B=128 96.2 / 77.3 / 70.5 / 70.8; floats, whose workgroups are more
 // at once (seven a CU, doubles five), with many values a tile, 2^24 REL 1e-2
-// B=16: 78.0 / 65.7 / 79.3 / 80.0.
+// B=16: 78.0 / 65.7 / 79.3 / 80.0.  256 against 512 KiB of values: 2^25 doubles
+// (sinusoids, REL 1e-3) B=16 154 / 217, B=128 135 / 150; against 128 KiB: 2^26
+// floats of the kind within 4 % either way.
 inline bool fused_shape(const Geom &g, uint64_t len, FusedShape *f)
 {
     if (g.B < kFusedMinB || g.B > kFusedMaxB || g.n == 0) return false;
@@ -601,7 +603,7 @@ inline bool fused_shape(const Geom &g, uint64_t len, FusedShape *f)
     uint64_t S = kFusedMaxTile;
     while (S / 2 >= f->V && S > 1792 &&
            (len < S * 512 || (g.es == 4 && len < S * 1024 && (g.n / 8192) * S > len) ||
-            (g.n / 65536) * S > len))
+            (g.n / (262144 / g.es)) * S > len))
         S /= 2;
     f->S = (uint32_t)S;
     const uint32_t want = g.B >= 128 ? 3u : g.B >= 64 ? 7u : kFusedMaxSec;

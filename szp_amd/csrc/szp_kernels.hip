@@ -2983,12 +2983,14 @@ __global__ __launch_bounds__(kWG) void k_decode(const uint8_t *__restrict__ st, 
 // What bounds it: latency (a tile's phases follow one another: staging and
 // boundaries ~105, walk ~48, sums ~53, look-back ~50, writing ~80 us of the
 // 512^3 field at REL 1e-4, B = 128) at 28 waves per CU, and in the unpacking
-// VALU issue.  Against a parse kernel that writes every block's position,
+// VALU issue (2 332 VALU instructions a wave, the VALUs 63 % busy over the
+// whole kernel).  Against a parse kernel that writes every block's position,
 // followed by a decode kernel that reads the stream again and looks back for
-// its carry: 480 -> 335 us on that field, 312 -> 213 us on a 384^3 float64
-// field (REL 1e-2, B = 64), 183 -> 133 us in fastMode 2 (384^3), 89 -> 29 us on
-// 100 003 values (B = 32).  Tiles of 11 and 20 KiB: 386 and 348 us.  Values go
-// out non-temporal in float (345 -> 335 us; double 213 -> 507 us).
+// its carry: 480 -> 335 us on that field, 312 -> 158 us on a 384^3 float64
+// field (REL 1e-2, B = 64; 213 before store_wave), 183 -> 132 us in fastMode 2
+// (384^3), 89 -> 28 us on 100 003 values (B = 32).  Tiles of 11 and 20 KiB: 386
+// and 348 us.  Values go out non-temporal in float (345 -> 335 us, although 4
+// bytes off their lines they are then written 1.18 times; double 213 -> 507 us).
 
 constexpr uint32_t kFusedSeg = 512;  // blocks whose positions are listed at a time
 
@@ -4414,11 +4416,14 @@ uint64_t decompress_workspace_bytes(uint64_t stream_bytes, uint64_t n, int B, in
 {
     Geom g;
     if (!make_geom(n, B, T, &g, 4, (uint32_t)mode)) return 0;
-    const uint64_t two = decompress_ws_layout(g, stream_bytes, nullptr, nullptr);
-    FusedShape f;
-    return fused_shape(g, stream_bytes, &f)
-               ? std::max(two, fused_ws_layout(g, f, stream_bytes, nullptr, nullptr))
-               : two;
+    uint64_t need = decompress_ws_layout(g, stream_bytes, nullptr, nullptr);
+    // The query knows no value type, and the fused tiles depend on it.
+    for (uint32_t es = 4; es <= 8; es += 4) {
+        FusedShape f;
+        if (make_geom(n, B, T, &g, es, (uint32_t)mode) && fused_shape(g, stream_bytes, &f))
+            need = std::max(need, fused_ws_layout(g, f, stream_bytes, nullptr, nullptr));
+    }
+    return need;
 }
 
 uint32_t *workspace_error_word(void *d_work)
